@@ -738,12 +738,15 @@ void reset_grid(mpm_ctx* ctx) {
   launch_fill_int(ctx->gflag, ctx->nblocks, 0, s);
   launch_fill_int(ctx->gcnt, 4, 0, s);
   launch_fill_int(ctx->dstep, 2, 1, s);
+  // the epochs start again in a binning made before: BV_STEP is of the old
+  // count, and with the velocities cleared no block is due for zeroing
+  launch_fill_int(ctx->bvars + BV_STEP, 1, 0, s);
   ctx->gacc_clean = true;
 }
 
 // One substep: re-bin when due, then the block pass (PASS_P2G on the first
-// substep of a call, PASS_FUSED after it), which advances the epoch at its
-// end, and the grid pass.
+// substep of a call, PASS_FUSED after it), and the grid pass, which advances
+// the epoch.
 int substep(mpm_ctx* ctx, float dt, bool first) {
   int rc;
   if (ctx->since_sort < 0 || ctx->since_sort >= ctx->resort_every)

@@ -75,7 +75,8 @@ struct BaseList {
   int* list[2];  // the current binning's blocks and the ones before it
   int* vars;     // BV_EPOCH: binnings so far; BV_CUR: which list is current;
                  // BV_STEP: substep epoch whose grid pass zeroes the blocks
-                 // that only the other list holds; BV_COUNT: lengths (2)
+                 // that only the other list holds (0: none, epochs are > 0;
+                 // set where the epochs start again); BV_COUNT: lengths (2)
 };
 
 // One scene: its grid (dims, spacing, place in the shared grid arrays), its
