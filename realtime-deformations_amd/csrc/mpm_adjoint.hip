@@ -126,8 +126,9 @@ __device__ __forceinline__ bool svd_of(const M3& F, M3& Lb, float (&s)[3], M3& R
 // launch for each part, and one that reset the map and the nodes of the
 // listed blocks after every substep, 48 reversed substeps of 3 x 20,011
 // particles spent 11 us each on it; the launches are 3 to 6 us a piece.)
-__global__ void __launch_bounds__(TPB) k_adj_nodes(KArgs a, GridRec done, float4* gdone, GridRec next, float4* gnext,
-                                                   float4* vnode) {
+// sdone, snext (null: gdone, gnext): FP64 sums of the velocity adjoints.
+__global__ void __launch_bounds__(TPB) k_adj_nodes(KArgs a, GridRec done, float4* gdone, const double4* sdone,
+                                                   GridRec next, float4* gnext, double4* snext, float4* vnode) {
   const int lane = threadIdx.x & 63;
   const int cnt = done.list ? done.list[0] : 0;
   const int total = cnt + (next.list ? next.list[0] : 0);
@@ -150,13 +151,22 @@ __global__ void __launch_bounds__(TPB) k_adj_nodes(KArgs a, GridRec done, float4
       i = bi * 4 + (lane >> 4), j = bj * 4 + ((lane >> 2) & 3), k = bk * 4 + (lane & 3);
     }
     if (!dn) {
-      gnext[g] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (snext)
+        snext[g] = make_double4(0.0, 0.0, 0.0, 0.0);
+      else
+        gnext[g] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (acc.x != 0.0f && (S.bc_mode & MPM_BC_DOMAIN))
         vpre = domain_walls(i, j, k, S.dims[0], S.dims[1], S.dims[2], vpre);
       vnode[g] = make_float4(vpre.x, vpre.y, vpre.z, 0.f);
       continue;
     }
-    const float4 gn = gdone[g];
+    float4 gn;
+    if (sdone) {
+      const double4 d = sdone[g];
+      gn = make_float4(0.f, (float)d.y, (float)d.z, (float)d.w);
+    } else {
+      gn = gdone[g];
+    }
     if (acc.x == 0.0f) {
       gdone[g] = make_float4(0.f, 0.f, 0.f, 0.f);
       continue;
@@ -482,9 +492,9 @@ __global__ void __launch_bounds__(TPB) k_rows_to_aos(float* dst, const float* sr
 
 // one wave per listed grid block, up to 2048 workgroups of 4 waves
 inline int rec_grid(const KArgs& a) { return (int)std::max<int64_t>(1, std::min<int64_t>((a.nnodes / 64 + 3) / 4, 2048)); }
-void launch_adj_nodes(const KArgs& a, const GridRec& done, float4* gdone, const GridRec& next, float4* gnext,
-                      float4* vnode, hipStream_t s) {
-  k_adj_nodes<<<rec_grid(a), TPB, 0, s>>>(a, done, gdone, next, gnext, vnode);
+void launch_adj_nodes(const KArgs& a, const GridRec& done, float4* gdone, const double4* sdone, const GridRec& next,
+                      float4* gnext, double4* snext, float4* vnode, hipStream_t s) {
+  k_adj_nodes<<<rec_grid(a), TPB, 0, s>>>(a, done, gdone, sdone, next, gnext, snext, vnode);
 }
 void launch_adj_p2g(const KArgs& a, const float* St, const float* Gin, float* Gout, const float4* gnode, float* gE,
                     const float* Sv, const float* SvPrev, hipStream_t s) {

@@ -10,8 +10,8 @@ enum AdjField : int { AX = FX, AV = FV, AB = FB, AFE = FFE, AFP = FFP, NA = FM }
 
 // the node work after the reverse G2P of one substep (done) and before that
 // of the next to be reversed; a null list skips either
-void launch_adj_nodes(const KArgs& a, const GridRec& done, float4* gdone, const GridRec& next, float4* gnext,
-                      float4* vnode, hipStream_t s);
+void launch_adj_nodes(const KArgs& a, const GridRec& done, float4* gdone, const double4* sdone, const GridRec& next,
+                      float4* gnext, double4* snext, float4* vnode, hipStream_t s);
 void launch_adj_p2g(const KArgs& a, const float* St, const float* Gin, float* Gout, const float4* gnode, float* gE,
                     const float* Sv, const float* SvPrev, hipStream_t s);
 // row transfers: slot order (pid: caller index per slot) <-> caller order

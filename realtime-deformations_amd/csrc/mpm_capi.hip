@@ -265,6 +265,7 @@ KArgs make_args(const mpm_ctx* c, float dt) {
   a.sc = c->scenes[0];
   a.status = c->status;
   a.exact = c->exact ? 1 : 0;
+  a.wide = a.exact;
   return a;
 }
 void host_collider_inverse(const float t[3], const float q[4], float inv[4][4]) {
@@ -431,7 +432,7 @@ int mpm_create_batch(const mpm_params* params, const int32_t* n_particles, int32
   alloc(&ctx->gcnt, sizeof(int) * 4);
   alloc(&ctx->dstep, 2 * sizeof(int));
   alloc(&ctx->bctr, sizeof(int));
-  alloc(&ctx->gacc, 2 * gbytes);  // a double4 per node (reproducible mode)
+  alloc(&ctx->gacc, 2 * gbytes);  // a double4 per node
   alloc(&ctx->gvel, gbytes);
   alloc(&ctx->gforce, gbytes);
   alloc(&ctx->status, sizeof(int) * nscenes);
@@ -505,7 +506,8 @@ int mpm_destroy(mpm_ctx* ctx) {
   }
   {
     const mpm_ctx::AdjWork& w = ctx->adj_ws;
-    void* b[] = {w.Gc, w.Gs, w.Gs2, w.gEs, w.gEc, w.tmp, w.gnode[0], w.gnode[1], w.vnode, w.seg, w.gsave, w.glist, w.svd};
+    void* b[] = {w.Gc,      w.Gs,      w.Gs2,   w.gEs, w.gEc,   w.tmp,   w.gnode[0],
+                 w.gnode[1], w.gsum[0], w.gsum[1], w.vnode, w.seg, w.gsave, w.glist, w.svd};
     for (void* q : b) (void)hipFree(q);
   }
   for (hipEvent_t e : ctx->events) (void)hipEventDestroy(e);
@@ -670,6 +672,7 @@ BaseList base_list(const mpm_ctx* ctx) { return BaseList{ctx->gbase, {ctx->base[
 BlockArgs block_args(mpm_ctx* ctx, float dt) {
   BlockArgs ba{};
   ba.a = make_args(ctx, dt);
+  if (ctx->chunk) ba.a.wide = 1;
   ba.blist = ctx->work;
   ba.nblk = ctx->nwork;
   ba.spread = ctx->chunk != 0;
@@ -1236,9 +1239,10 @@ int record_segment(mpm_ctx* ctx, float dt, int ns, float* seg, float4* gs, int* 
   if (!ctx->gacc_clean) reset_grid(ctx);
   for (int k = 0; k < ns; ++k) {
     BlockArgs ba = block_args(ctx, dt);
-    // the recording passes sum in the default (FP32) format, so the grid
-    // pass must read that format in reproducible mode too
+    // the recording passes do not sum on the quanta, so the grid pass must
+    // read the default mode's format in reproducible mode too
     ba.a.exact = 0;
+    ba.a.wide = ctx->chunk != 0;
     ba.rec = seg + (size_t)k * NA * sd;
     ba.rec_svd = sv + (size_t)k * SVD_ROWS * sd;
     ba.grec = grid_record(ctx, gs, gl, k);
@@ -1285,7 +1289,12 @@ int adjoint_workspace(mpm_ctx* ctx, int every) {
   alloc(&w.gEc, sizeof(float) * sd);
   alloc(&w.tmp, sizeof(float) * 3 * (size_t)std::max(1, ctx->n));
   alloc(&w.gnode[0], sizeof(float4) * (size_t)ctx->nnodes);
-  alloc(&w.gnode[1], sizeof(float4) * (size_t)ctx->nnodes);
+  if (ctx->chunk) {
+    alloc(&w.gsum[0], sizeof(double4) * (size_t)ctx->nnodes);
+    alloc(&w.gsum[1], sizeof(double4) * (size_t)ctx->nnodes);
+  } else {
+    alloc(&w.gnode[1], sizeof(float4) * (size_t)ctx->nnodes);
+  }
   alloc(&w.vnode, sizeof(float4) * (size_t)ctx->nnodes);
   if (every > 1 && every > w.seg_every) {
     // states of a segment's substeps plus the positions after it; the grid
@@ -1310,8 +1319,8 @@ int adjoint_workspace(mpm_ctx* ctx, int every) {
   return MPM_OK;
 }
 
-// w.gnode[k & 1] holds the node adjoints of substep k, w.vnode its node
-// velocities.
+// w.gnode[k & 1], or with parts of blocks w.gsum[k & 1] and then w.gnode[0],
+// holds the node adjoints of substep k, w.vnode its node velocities.
 void adjoint_segment(mpm_ctx* ctx, float dt, int ns, const float* seg, float4* gs, int* gl, const float* sv,
                      float*& Gs, float*& Gs2, float* gEs) {
   const int64_t sd = ctx->stride;
@@ -1319,18 +1328,18 @@ void adjoint_segment(mpm_ctx* ctx, float dt, int ns, const float* seg, float4* g
   mpm_ctx::AdjWork& w = ctx->adj_ws;
   const GridRec none{nullptr, nullptr};
   GridRec cur = grid_record(ctx, gs, gl, ns - 1);
-  launch_adj_nodes(make_args(ctx, dt), none, nullptr, cur, w.gnode[(ns - 1) & 1], w.vnode, s);
+  auto gnode = [&](int k) { return w.gnode[ctx->chunk ? 0 : k & 1]; };
+  auto gsum = [&](int k) { return w.gsum[k & 1]; };
+  launch_adj_nodes(make_args(ctx, dt), none, nullptr, nullptr, cur, gnode(ns - 1), gsum(ns - 1), w.vnode, s);
   for (int k = ns - 1; k >= 0; --k) {
     const float* St = seg + (size_t)k * NA * sd;
     const float* Xn = seg + (size_t)(k + 1) * NA * sd;
-    float4* gnode = w.gnode[k & 1];
-    BlockArgs ba = block_args(ctx, dt);
-    ba.grec = cur;
-    launch_adj_g2p_block(ba, St, Xn, Gs, Gs2, gnode, w.vnode, s);
+    const BlockArgs ba = block_args(ctx, dt);
+    launch_adj_g2p_block(ba, St, Xn, Gs, Gs2, gnode(k), gsum(k), w.vnode, s);
     const GridRec next = k > 0 ? grid_record(ctx, gs, gl, k - 1) : none;
-    launch_adj_nodes(ba.a, cur, gnode, next, w.gnode[(k + 1) & 1], w.vnode, s);
+    launch_adj_nodes(ba.a, cur, gnode(k), gsum(k), next, gnode(k + 1), gsum(k + 1), w.vnode, s);
     const float* Sv = sv + (size_t)k * SVD_ROWS * sd;
-    launch_adj_p2g(ba.a, St, Gs, Gs2, gnode, gEs, Sv, k > 0 ? Sv - (size_t)SVD_ROWS * sd : nullptr, s);
+    launch_adj_p2g(ba.a, St, Gs, Gs2, gnode(k), gEs, Sv, k > 0 ? Sv - (size_t)SVD_ROWS * sd : nullptr, s);
     std::swap(Gs, Gs2);
     cur = next;
   }

@@ -327,8 +327,8 @@ __device__ __forceinline__ void scatter_one(const BlockArgs& ba, const Scene& S,
 }
 
 // The global-memory scatter of a particle whose stencil left its block's
-// halo: atomics into the grid accumulators (FP32, or FP64 on the quanta in
-// reproducible mode), touched grid blocks marked.
+// halo: atomics into the grid accumulators (in reproducible mode on the
+// quanta), touched grid blocks marked.
 template <int EXACT>
 __device__ __forceinline__ void scatter_global(const BlockArgs& ba, const Scene& S, const StencilInfo& s, F3 x, float m,
                                             F3 mv, const M3& Q) {
@@ -350,6 +350,12 @@ __device__ __forceinline__ void scatter_global(const BlockArgs& ba, const Scene&
         atomicAdd(g + 1, on_quantum((double)px, Mp));
         atomicAdd(g + 2, on_quantum((double)py, Mp));
         atomicAdd(g + 3, on_quantum((double)pz, Mp));
+      } else if (a.wide) {
+        double* g = reinterpret_cast<double*>(a.gacc64 + gi);
+        atomicAdd(g + 0, (double)vm);
+        atomicAdd(g + 1, (double)px);
+        atomicAdd(g + 2, (double)py);
+        atomicAdd(g + 3, (double)pz);
       } else {
         float* g = reinterpret_cast<float*>(a.gacc + gi);
         atomicAdd(g + 0, vm);
@@ -577,7 +583,7 @@ __global__ void __launch_bounds__(TPB, 3) k_block_pass(BlockArgs ba) {
       for (int q = t; q < HN * HN * HN; q += TPB) {
         const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
         const int l = hx * TX + tile_y(hy) + tile_z(hz);
-        if (EXACT) {  // exact FP64 sums of multiples of the quanta
+        if (EXACT || a.wide) {  // EXACT: exact sums of multiples of the quanta
           const double m = ah[l], px = ah[TPLANE + l], py = ah[2 * TPLANE + l], pz = ah[3 * TPLANE + l];
           if (m != 0.0 || px != 0.0 || py != 0.0 || pz != 0.0) {
             const int gi = o[0] + hx, gj = o[1] + hy, gk = o[2] + hz;
@@ -619,7 +625,7 @@ template <int BATCHED>
 __global__ void __launch_bounds__(TPB) k_adj_g2p_block(BlockArgs ba, const float* __restrict__ St,
                                                        const float* __restrict__ Xn, const float* __restrict__ Gin,
                                                        float* __restrict__ Gout, float4* __restrict__ gnode,
-                                                       const float4* __restrict__ vnode) {
+                                                       double4* __restrict__ gsum, const float4* __restrict__ vnode) {
   __shared__ float vh[3 * PLANE];
   __shared__ double gh[3 * TPLANE];  // tiled like the forward accumulators
   __shared__ int claimed;
@@ -778,10 +784,17 @@ __global__ void __launch_bounds__(TPB) k_adj_g2p_block(BlockArgs ba, const float
               const int64_t g = node_index(i, j, k, S);
               const float4 vn = vnode[g];
               const F3 wu = node(ia, ib, ic, f3(vn.x, vn.y, vn.z));
-              float* gn = reinterpret_cast<float*>(gnode + g);
-              atomicAdd(gn + 1, wu.x);
-              atomicAdd(gn + 2, wu.y);
-              atomicAdd(gn + 3, wu.z);
+              if (gsum) {
+                double* gn = reinterpret_cast<double*>(gsum + g);
+                atomicAdd(gn + 1, (double)wu.x);
+                atomicAdd(gn + 2, (double)wu.y);
+                atomicAdd(gn + 3, (double)wu.z);
+              } else {
+                float* gn = reinterpret_cast<float*>(gnode + g);
+                atomicAdd(gn + 1, wu.x);
+                atomicAdd(gn + 2, wu.y);
+                atomicAdd(gn + 3, wu.z);
+              }
             }
       }
 #pragma unroll
@@ -791,14 +804,22 @@ __global__ void __launch_bounds__(TPB) k_adj_g2p_block(BlockArgs ba, const float
     for (int q = t; q < HN * HN * HN; q += TPB) {
       const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
       const int l = hx * TX + tile_y(hy) + tile_z(hz);
-      const float u0 = (float)gh[l], u1 = (float)gh[TPLANE + l], u2 = (float)gh[2 * TPLANE + l];
-      if (u0 != 0.0f || u1 != 0.0f || u2 != 0.0f) {
+      const double u0 = gh[l], u1 = gh[TPLANE + l], u2 = gh[2 * TPLANE + l];
+      if (u0 != 0.0 || u1 != 0.0 || u2 != 0.0) {
         const int gi = o[0] + hx, gj = o[1] + hy, gk = o[2] + hz;
         if (gi >= 0 && gj >= 0 && gk >= 0 && gi < S.dims[0] && gj < S.dims[1] && gk < S.dims[2]) {
-          float* gn = reinterpret_cast<float*>(gnode + node_index(gi, gj, gk, S));
-          atomicAdd(gn + 1, u0);
-          atomicAdd(gn + 2, u1);
-          atomicAdd(gn + 3, u2);
+          const int64_t g = node_index(gi, gj, gk, S);
+          if (gsum) {
+            double* gn = reinterpret_cast<double*>(gsum + g);
+            atomicAdd(gn + 1, u0);
+            atomicAdd(gn + 2, u1);
+            atomicAdd(gn + 3, u2);
+          } else {
+            float* gn = reinterpret_cast<float*>(gnode + g);
+            atomicAdd(gn + 1, (float)u0);
+            atomicAdd(gn + 2, (float)u1);
+            atomicAdd(gn + 3, (float)u2);
+          }
         }
       }
     }
@@ -841,7 +862,7 @@ template <int BATCHED> __global__ void __launch_bounds__(TPB) k_grid_active(Bloc
       // an FP32 zero)
       bool touched;
       float4 acc;
-      if (a.exact) {
+      if (a.wide) {
         const double4 d = a.gacc64[g];
         acc = make_float4((float)d.x, (float)d.y, (float)d.z, (float)d.w);
         touched = d.x != 0.0 || d.y != 0.0 || d.z != 0.0 || d.w != 0.0;
@@ -930,11 +951,11 @@ void launch_block_pass(const BlockArgs& ba, int mode, hipStream_t s) {
 }
 
 void launch_adj_g2p_block(const BlockArgs& ba, const float* St, const float* Xn, const float* Gin, float* Gout,
-                          float4* gnode, const float4* vnode, hipStream_t s) {
+                          float4* gnode, double4* gsum, const float4* vnode, hipStream_t s) {
   if (ba.a.nscenes == 1)
-    k_adj_g2p_block<0><<<ba.grid, TPB, 0, s>>>(ba, St, Xn, Gin, Gout, gnode, vnode);
+    k_adj_g2p_block<0><<<ba.grid, TPB, 0, s>>>(ba, St, Xn, Gin, Gout, gnode, gsum, vnode);
   else
-    k_adj_g2p_block<1><<<ba.grid, TPB, 0, s>>>(ba, St, Xn, Gin, Gout, gnode, vnode);
+    k_adj_g2p_block<1><<<ba.grid, TPB, 0, s>>>(ba, St, Xn, Gin, Gout, gnode, gsum, vnode);
 }
 
 void launch_grid_active(const BlockArgs& ba, hipStream_t s) {

@@ -53,9 +53,10 @@ constexpr int SVD_ROWS = 21;
 // accumulated in an FP64 LDS halo, flushed with one set of global atomics per
 // block.  St: stored state of the substep (slot order); Xn: rows holding the
 // next state's positions; Gin: the adjoints of the next state; Gout.x receives
-// the partial position adjoint; gnode.yzw the node adjoints.
+// the partial position adjoint; gnode.yzw the node adjoints, or gsum.yzw (not
+// null) with parts of blocks, whose sums are not to be rounded part by part.
 void launch_adj_g2p_block(const BlockArgs& ba, const float* St, const float* Xn, const float* Gin, float* Gout,
-                          float4* gnode, const float4* vnode, hipStream_t s);
+                          float4* gnode, double4* gsum, const float4* vnode, hipStream_t s);
 void launch_block_pass(const BlockArgs& ba, int mode, hipStream_t s);
 void launch_grid_active(const BlockArgs& ba, hipStream_t s);
 

@@ -108,8 +108,8 @@ struct KArgs {
   float* P;
   int64_t stride;
   int n;           // particles over all scenes
-  float4* gacc;    // (m, p) accumulators, FP32 (default mode)
-  double4* gacc64; // the same memory as FP64 accumulators (reproducible mode)
+  float4* gacc;    // (m, p) accumulators, FP32
+  double4* gacc64; // the same memory as FP64 accumulators (with wide)
   float4* gvel;    // (v, m) after the grid update
   float4* gforce;  // (f, 0), legacy stage path only
   int64_t nnodes;  // nodes over all scenes
@@ -121,6 +121,11 @@ struct KArgs {
   Scene sc;              // scene 0 by value (legacy stage kernels: one scene)
   int* status;           // per scene
   int exact;             // reproducible mode (P2G sums on the scenes' quanta)
+  // FP64 accumulators: reproducible mode, and block passes over parts of
+  // blocks.  A whole block's sums are rounded to FP32 once, where its halo is
+  // flushed; of a block in parts, hundreds of them where it is crowded, each
+  // would be rounded on its own and the FP32 sum of them again at every add.
+  int wide;
 };
 
 // Reproducible P2G sums.  M = quantum_magic(k) = 1.5 * 2^(52 + k); for
@@ -133,9 +138,9 @@ struct KArgs {
 __device__ __forceinline__ double quantum_magic(int k) { return ldexp(1.5, 52 + k); }
 __device__ __forceinline__ double on_quantum(double c, double M) { return (c + M) - M; }
 
-// P2G sums of node g as FP32, from the accumulators of the mode
+// P2G sums of node g as FP32, from the accumulators in use
 __device__ __forceinline__ float4 load_acc(const KArgs& a, int64_t g) {
-  if (a.exact) {
+  if (a.wide) {
     const double4 d = a.gacc64[g];
     return make_float4((float)d.x, (float)d.y, (float)d.z, (float)d.w);
   }
@@ -201,8 +206,8 @@ struct mpm_ctx {
   int since_sort = -1;      // substeps since the last binning (-1: never binned)
   int resort_every = 16;
   int block_grid = 2048;    // workgroups of the persistent block pass
-  double4* gacc = nullptr;  // (m, p) accumulators: FP64 in reproducible mode,
-                            // else FP32 in the first half
+  double4* gacc = nullptr;  // (m, p) accumulators: FP64 with KArgs.wide, else
+                            // FP32 in the first half
   float4* gvel = nullptr;
   float4* gforce = nullptr;
   int* status = nullptr;    // device status word per scene
@@ -265,7 +270,10 @@ struct mpm_ctx {
   // reverse-sweep workspaces, kept between calls (freed by mpm_destroy)
   struct AdjWork {
     float *Gc = nullptr, *Gs = nullptr, *Gs2 = nullptr, *gEs = nullptr, *gEc = nullptr, *tmp = nullptr;
-    float4* gnode[2] = {nullptr, nullptr};  // node adjoints, by parity of the substep
+    // node adjoints, by parity of the substep: gnode itself, or with parts of
+    // blocks (chunk > 0) FP64 sums in gsum and what becomes of them in gnode[0]
+    float4* gnode[2] = {nullptr, nullptr};
+    double4* gsum[2] = {nullptr, nullptr};
     float4* vnode = nullptr;  // node velocities of the substep being reversed
     float* seg = nullptr;     // (every + 1) x 33 rows
     float4* gsave = nullptr;  // every x nnodes
