@@ -3,6 +3,7 @@
 // and the deformation-gradient update to the oracle bit for bit.  Built as
 // lib/libmpm_hostcheck.so; not part of libmpm_hip.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 
 #include "mpm_hostutil.hpp"
@@ -66,6 +67,17 @@ int hc_svd3(const float* M, float* U, float* S, float* V) {
       V[3 * r + c] = v[r][c];
     }
   return ok ? 0 : 1;
+}
+
+// the Jacobi SVD's scaling: W[i] = M[i] / max |M[i]| of n matrices
+void hc_scale_down(const float* M, int n, float* W) {
+  for (int i = 0; i < n; ++i) {
+    float m[3][3], w[3][3], scale = 0.0f;
+    std::memcpy(m, M + 9 * i, sizeof m);
+    for (int k = 0; k < 9; ++k) scale = std::max(scale, std::fabs(M[9 * i + k]));
+    scale_down(m, scale, w);
+    std::memcpy(W + 9 * i, w, sizeof w);
+  }
 }
 
 // glm column-major matrices; returns 0, or 1 when the SVD rejects its input

@@ -234,7 +234,9 @@ MPM_HD void scale_down(const float (&M)[3][3], float scale, float (&W)[3][3]) {
   float lo = fabsf(M[0][0]);
 #pragma unroll
   for (int k = 1; k < 9; ++k) lo = fminf(lo, fabsf(M[k / 3][k % 3]));
-  if (lo >= 8.27180613e-25f && scale <= 1.20892582e24f) {  // 2^-80, 2^80: every quotient is normal
+  // entries of 2^-80 to 2^20: quotients of 2^-100 or more (in the subnormal
+  // range the correction would not round like a division)
+  if (lo >= 8.27180613e-25f && scale <= 1048576.0f) {
     const float r = rcp_exact(scale);
 #pragma unroll
     for (int k = 0; k < 9; ++k) W[k / 3][k % 3] = div_exact(M[k / 3][k % 3], scale, r);

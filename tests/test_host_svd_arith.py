@@ -1,0 +1,56 @@
+"""The Jacobi SVD's short quotients, from the library's math source built for
+the host (their reciprocals and roots correctly rounded there), bit for bit
+against IEEE division where they hand over to it."""
+import ctypes as C
+import os
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "realtime-deformations_amd", "lib", "libmpm_hostcheck.so")
+_F = C.POINTER(C.c_float)
+
+
+@pytest.fixture(scope="module")
+def hc():
+    if not os.path.exists(LIB):
+        pytest.fail(f"{LIB} missing: run realtime-deformations_amd/build.py")
+    L = C.CDLL(LIB)
+    L.hc_scale_down.argtypes = [_F, C.c_int, _F]
+    return L
+
+
+def _scaled(hc, M):
+    W = np.empty_like(M)
+    hc.hc_scale_down(M.ctypes.data_as(_F), M.shape[0], W.ctypes.data_as(_F))
+    return W
+
+
+def _ties(rng, n):
+    """Matrices whose quotients lie half-way between two subnormal numbers:
+    entries a = (2 k + 1) 2^-150 b beside their largest, b, of 12 bits."""
+    b = (rng.integers(1 << 11, 1 << 12, n) * 2.0 ** -11)[:, None]
+    eb = rng.integers(55, 81, (n, 1))
+    a = (2 * rng.integers(1, 1 << 11, (n, 8)) + 1) * 2.0 ** -150 * b * 2.0 ** eb
+    M = np.concatenate([b * 2.0 ** eb, a], 1) * rng.choice([-1.0, 1.0], (n, 9))
+    assert (np.float32(M).astype(np.float64) == M).all()
+    return np.float32(M)
+
+
+def _spread(rng, n, lo, hi):
+    return np.float32(rng.choice([-1.0, 1.0], (n, 9)) * 2.0 ** rng.uniform(lo, hi, (n, 9)))
+
+
+@pytest.mark.parametrize("kind", ["ties", "2^-79 to 2^79", "around 2^-80", "around 2^20", "around 2^80", "near 1"])
+def test_scaled_entries_round_like_ieee_division(hc, kind):
+    rng = np.random.default_rng(7)
+    n = 200000
+    M = {"ties": lambda: _ties(rng, n),
+         "2^-79 to 2^79": lambda: _spread(rng, n, -79, 79),
+         "around 2^-80": lambda: _spread(rng, n, -82, -70),
+         "around 2^20": lambda: _spread(rng, n, -80, 21),
+         "around 2^80": lambda: _spread(rng, n, 60, 82),
+         "near 1": lambda: _spread(rng, n, -30, 1)}[kind]()
+    scale = np.abs(M).max(axis=1, keepdims=True)
+    np.testing.assert_array_equal(_scaled(hc, M).view(np.uint32), (M / scale).view(np.uint32))
