@@ -80,6 +80,11 @@ void hc_scale_down(const float* M, int n, float* W) {
   }
 }
 
+// (1 / w, u / w), w = sqrt(1 + u^2), as a rotation takes them
+void hc_rcp_pair(const float* u, int n, float* rw, float* uw) {
+  for (int i = 0; i < n; ++i) rcp_pair(u[i], sqrt_ge1(1.0f + u[i] * u[i]), rw[i], uw[i]);
+}
+
 // glm column-major matrices; returns 0, or 1 when the SVD rejects its input
 int hc_fupdate(int compose, float dt, float h, double theta_c, double theta_s, const float* B, const float* FE,
                const float* FP, float* FEo, float* FPo) {

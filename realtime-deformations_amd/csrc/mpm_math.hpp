@@ -216,7 +216,8 @@ MPM_HD double rcp_unit(double y) { return 1.0 / y; }
 MPM_HD void rcp_pair(float u, float w, float& rw, float& uw) {
   if (fabsf(u) <= 1.15292150e18f) {  // 2^60
     rw = rcp_exact(w);
-    uw = div_exact(u, w, rw);  // |u| < 2^-60: w = 1, exact as it is
+    // |u| < 2^-60: w = 1, exact as it is, but for the sign of -0
+    uw = __builtin_copysignf(div_exact(u, w, rw), u);
   } else {
     rw = 1.0f / w;
     uw = u / w;
