@@ -347,6 +347,12 @@ int mpm_debug_bin(mpm_ctx* ctx, uint32_t* sorted_keys, uint32_t* perm, int32_t* 
  * count). */
 int mpm_debug_blocks(mpm_ctx* ctx, int32_t* blocks, int32_t max_blocks, int32_t* count);
 
+/* The device arithmetic of the F update's Jacobi SVD (no reference
+ * counterpart) on n values: out[k] = 1 / a[k] (op 0), a[k] / b[k] (op 1) or
+ * sqrt(a[k]) for a[k] >= 1 (op 2), as a rotation computes them; b is read by
+ * op 1 only. */
+int mpm_debug_svd_arith(mpm_ctx* ctx, int32_t op, const float* a, const float* b, int32_t n, float* out);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1565,6 +1565,31 @@ extern "C" int mpm_debug_blocks(mpm_ctx* ctx, int32_t* blocks, int32_t max_block
 }
 
 namespace {
+__global__ void __launch_bounds__(256) k_svd_arith(int op, const float* a, const float* b, int n, float* out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  out[i] = op == 0 ? rcp_exact(a[i]) : op == 1 ? div_exact(a[i], b[i], rcp_exact(b[i])) : sqrt_ge1(a[i]);
+}
+}  // namespace
+
+extern "C" int mpm_debug_svd_arith(mpm_ctx* ctx, int32_t op, const float* a, const float* b, int32_t n, float* out) {
+  if (check_ctx(ctx) || op < 0 || op > 2 || n < 0 || (n && (!a || !out || (op == 1 && !b)))) return MPM_ERR_ARG;
+  if (n == 0) return MPM_OK;
+  const size_t bytes = sizeof(float) * (size_t)n;
+  DevBuf<float> da, db, dout;
+  MPM_HIP(da.alloc(bytes));
+  MPM_HIP(db.alloc(bytes));
+  MPM_HIP(dout.alloc(bytes));
+  MPM_HIP(hipMemcpyAsync(da.p, a, bytes, hipMemcpyHostToDevice, ctx->stream));
+  if (op == 1) MPM_HIP(hipMemcpyAsync(db.p, b, bytes, hipMemcpyHostToDevice, ctx->stream));
+  k_svd_arith<<<(n - 1) / 256 + 1, 256, 0, ctx->stream>>>(op, da.p, db.p, n, dout.p);
+  MPM_HIP(hipGetLastError());
+  MPM_HIP(hipMemcpyAsync(out, dout.p, bytes, hipMemcpyDeviceToHost, ctx->stream));
+  MPM_HIP(hipStreamSynchronize(ctx->stream));
+  return MPM_OK;
+}
+
+namespace {
 __global__ void __launch_bounds__(256) k_copy_probe(const float4* __restrict__ src, float4* __restrict__ dst,
                                                     int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)

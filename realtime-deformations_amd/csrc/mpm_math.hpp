@@ -177,15 +177,16 @@ MPM_HD float div_rcp(float a, float b, float rb) {
 // root: scaling for denormals and infinities) were half of a Jacobi rotation.
 // On the ranges the rotations meet, shorter ones round the same:
 //  - rcp_exact(y), |y| in [2^-100, 2^100]: the hardware reciprocal (1 ulp)
-//    and one Newton step.  Equal to 1 / y on every FP32 significand.
+//    and one Newton step.
 //  - div_exact(a, b, r), r = rcp_exact(b): the quotient a r is within 1.5 ulp
-//    and div_rcp's correction rounds it.  Equal to a / b on every pair whose
-//    quotient lies close enough to a rounding boundary for the correction's
-//    own error to matter, and on 5e8 others.  |a| and the quotient must stay
-//    above 2^-100 or so (or be 0), so that the residual is exact.
+//    and div_rcp's correction rounds it.  |a| and the quotient must stay
+//    above 2^-100 or so (or be 0), so that the residual is exact and the
+//    quotient normal.
 //  - sqrt_ge1(x), x >= 1 or infinite or NaN: the hardware root (1 ulp) and
-//    the residuals of its two neighbours.  Equal to sqrtf on every
-//    significand of both exponent parities.
+//    the residuals of its two neighbours.
+// tests/test_gpu_svd_arith.py holds them to IEEE results on the device: every
+// significand of the reciprocal, of both exponent parities of the root, and
+// quotients built as close to a rounding boundary as a pair allows.
 // Fused pass where the SVD rotates: 1,048,576 particles landing 202.6 ->
 // 195.2 us, 5,010,000 in 64 snowballs 596 -> 592; at rest (few rotations)
 // unchanged.

@@ -88,7 +88,8 @@ EXPORTS = [
     "mpm_default_params", "mpm_create", "mpm_destroy", "mpm_last_error", "mpm_num_particles",
     "mpm_set_particles", "mpm_set_state", "mpm_set_colliders", "mpm_init_volumes", "mpm_stage",
     "mpm_substeps", "mpm_sync", "mpm_get_particles", "mpm_get_grid", "mpm_profile_begin", "mpm_profile_end",
-    "mpm_count_active", "mpm_debug_bin", "mpm_debug_blocks", "mpm_copy_probe", "mpm_use_graphs",
+    "mpm_count_active", "mpm_debug_bin", "mpm_debug_blocks", "mpm_debug_svd_arith", "mpm_copy_probe",
+    "mpm_use_graphs",
     "mpm_set_reproducible", "mpm_get_reproducible",
     "mpm_create_batch", "mpm_num_scenes", "mpm_scene_set_particles", "mpm_scene_set_state",
     "mpm_scene_set_colliders", "mpm_scene_get_particles", "mpm_scene_get_grid", "mpm_scene_status",
@@ -147,6 +148,7 @@ def lib():
         L.mpm_count_active.argtypes = [vp, C.POINTER(C.c_int64)]
         L.mpm_debug_bin.argtypes = [vp, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32), C.POINTER(C.c_int32)]
         L.mpm_debug_blocks.argtypes = [vp, C.POINTER(C.c_int32), C.c_int32, C.POINTER(C.c_int32)]
+        L.mpm_debug_svd_arith.argtypes = [vp, C.c_int32, _F, _F, C.c_int32, _F]
         L.mpm_copy_probe.argtypes = [vp, C.c_int64]
         L.mpm_scene_generate.argtypes = [vp, C.c_int32, C.POINTER(Generator), C.POINTER(C.c_int64)]
         L.mpm_generate.argtypes = [vp, C.POINTER(Generator), C.POINTER(C.c_int64)]
@@ -333,6 +335,15 @@ class Simulation:
         if cnt.value:
             self._check(self.L.mpm_debug_blocks(self.ctx, out.ctypes.data_as(C.POINTER(C.c_int32)), cnt.value,
                                                 C.byref(cnt)))
+        return out
+
+    def debug_svd_arith(self, op, a, b=None):
+        """The Jacobi SVD's device arithmetic: "rcp" 1 / a, "div" a / b, "sqrt"
+        of a >= 1."""
+        a, b = _f32(a), _f32(b)
+        out = np.zeros_like(a)
+        self._check(self.L.mpm_debug_svd_arith(self.ctx, ("rcp", "div", "sqrt").index(op), _fp(a), _fp(b), a.size,
+                                               _fp(out)))
         return out
 
     def particles(self):
