@@ -122,4 +122,13 @@ void hc_readback_parts(size_t bytes, unsigned nt, size_t* begin, size_t* end) {
   }
 }
 
+// How a copy of `total` bytes to the caller is cut: threads, bytes per piece,
+// bytes of pinned memory.
+void hc_xfer_plan(size_t total, size_t out[3]) {
+  const XferPlan p = xfer_plan(total);
+  out[0] = p.threads;
+  out[1] = p.piece;
+  out[2] = p.ring;
+}
+
 }  // extern "C"

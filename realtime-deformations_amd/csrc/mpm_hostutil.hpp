@@ -1,6 +1,7 @@
 // Host-side helpers shared by libmpm_hip and its host check library (plain
 // C++, no HIP types).
 #pragma once
+#include <algorithm>
 #include <cstddef>
 
 namespace mpm {
@@ -12,6 +13,24 @@ namespace mpm {
 inline size_t readback_part_bytes(size_t bytes, unsigned nt) {
   const size_t per = (bytes + nt - 1) / nt;
   return (per + 63) / 64 * 64;
+}
+
+// A copy of `total` bytes to the caller through pinned memory: pieces of up to
+// 1 MiB, two in flight per host thread, up to four threads; `ring` bytes of
+// pinned memory hold the pieces in flight.
+struct XferPlan {
+  unsigned threads;
+  size_t piece, ring;
+};
+constexpr size_t XFER_PIECE = size_t(1) << 20, XFER_PIECE_MIN = size_t(1) << 17;
+constexpr unsigned XFER_THREADS = 4;
+inline XferPlan xfer_plan(size_t total) {
+  XferPlan p;
+  p.threads = (unsigned)std::min<size_t>(XFER_THREADS, std::max<size_t>(1, total / (2 * XFER_PIECE)));
+  p.piece = std::min(XFER_PIECE, std::max(XFER_PIECE_MIN, readback_part_bytes(total, 4 * p.threads)));
+  p.piece = std::min(p.piece, std::max<size_t>(64, readback_part_bytes(total, 1)));
+  p.ring = 2 * p.threads * p.piece;
+  return p;
 }
 
 }  // namespace mpm

@@ -285,6 +285,7 @@ struct mpm_ctx {
   int* st_host = nullptr;        // pinned: status words read back
   // readback: pinned pieces on the way to the caller's arrays
   char* xfer_host = nullptr;
+  size_t xfer_cap = 0;           // its bytes: what the largest read so far needed
   hipEvent_t xfer_ev[8] = {};
   // positions readback: device staging, pinned host mirror, copy stream
   float* pos_stage = nullptr;

@@ -235,15 +235,21 @@ void gather_positions(mpm_ctx* ctx, bool status) {
   launch_gather_fields(l, ctx->P, ctx->stride, ctx->pid, 0, ctx->n, ctx->stream);
 }
 
-// Pieces of a copy to the caller: up to 1 MiB, two in flight per host thread,
-// up to four threads.  A kernel writes a piece to pinned memory (a copy engine
-// takes 20 us to start, and pageable memory makes the runtime stage it
-// serially); the thread moves it on, which also touches the caller's pages.
-constexpr size_t PIECE = size_t(1) << 20, PIECE_MIN = size_t(1) << 17;
-constexpr unsigned XFER_THREADS = 4;
-
-int ensure_xfer(mpm_ctx* ctx, bool ring) {
-  if (ring && !ctx->xfer_host) IO_HIP(hipHostMalloc(&ctx->xfer_host, PIECE * 2 * XFER_THREADS));
+// What a copy to the caller needs: events, and without a mirror `ring` bytes of
+// pinned memory.  A kernel writes a piece to pinned memory (a copy engine takes
+// 20 us to start, and pageable memory makes the runtime stage it serially); a
+// host thread moves it on, which also touches the caller's pages.
+int ensure_xfer(mpm_ctx* ctx, size_t ring) {
+  if (ctx->xfer_cap < ring) {
+    if (ctx->xfer_host) {
+      IO_HIP(hipStreamSynchronize(ctx->stream));
+      IO_HIP(hipHostFree(ctx->xfer_host));
+      ctx->xfer_host = nullptr;
+      ctx->xfer_cap = 0;
+    }
+    IO_HIP(hipHostMalloc(&ctx->xfer_host, ring));
+    ctx->xfer_cap = ring;
+  }
   for (hipEvent_t& e : ctx->xfer_ev)
     if (!e) IO_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   return MPM_OK;
@@ -270,8 +276,9 @@ int copy_to_host(mpm_ctx* ctx, const XferPart* parts, int count, char* mirror) {
   std::vector<Piece> pieces;
   size_t total = 0;
   for (int k = 0; k < count; ++k) total += parts[k].bytes;
-  const unsigned nt = (unsigned)std::min<size_t>(XFER_THREADS, std::max<size_t>(1, total / (2 * PIECE)));
-  const size_t piece = std::min(PIECE, std::max(PIECE_MIN, readback_part_bytes(total, 4 * nt)));
+  const XferPlan plan = xfer_plan(total);
+  const unsigned nt = plan.threads;
+  const size_t piece = plan.piece;
   size_t at = 0;
   for (int k = 0; k < count; ++k)
     for (size_t o = 0; o < parts[k].bytes; o += piece) {
@@ -284,7 +291,7 @@ int copy_to_host(mpm_ctx* ctx, const XferPart* parts, int count, char* mirror) {
     IO_HIP(hipStreamSynchronize(ctx->stream));
     return MPM_OK;
   }
-  if (int rc = ensure_xfer(ctx, !mirror)) return rc;
+  if (int rc = ensure_xfer(ctx, mirror ? 0 : plan.ring)) return rc;
   if (pieces.size() == 1) {  // nothing to overlap: one wait
     const Piece& p = pieces[0];
     char* via = p.via ? p.via : ctx->xfer_host;
@@ -305,7 +312,7 @@ int copy_to_host(mpm_ctx* ctx, const XferPart* parts, int count, char* mirror) {
       if (i < pieces.size()) {
         Piece& p = pieces[i];
         const unsigned slot = 2 * t + (k & 1);
-        if (!p.via) p.via = ctx->xfer_host + slot * PIECE;
+        if (!p.via) p.via = ctx->xfer_host + slot * piece;
         launch_copy_out(p.via, p.src, (int64_t)(p.bytes / 4), ctx->stream);
         if ((e = hipGetLastError()) == hipSuccess) e = hipEventRecord(ctx->xfer_ev[slot], ctx->stream);
       }
