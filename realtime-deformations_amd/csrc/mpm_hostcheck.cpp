@@ -131,4 +131,14 @@ void hc_xfer_plan(size_t total, size_t out[3]) {
   out[2] = p.ring;
 }
 
+// Number of pieces of a copy's parts, and piece i as (part, offset, bytes, at).
+size_t hc_xfer_pieces(const size_t* bytes, int count, size_t piece) { return xfer_pieces(bytes, count, piece); }
+void hc_xfer_piece(const size_t* bytes, int count, size_t piece, size_t i, size_t out[4]) {
+  const XferPiece p = xfer_piece(bytes, count, piece, i);
+  out[0] = (size_t)p.part;
+  out[1] = p.offset;
+  out[2] = p.bytes;
+  out[3] = p.at;
+}
+
 }  // extern "C"

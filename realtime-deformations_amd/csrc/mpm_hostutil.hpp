@@ -33,4 +33,28 @@ inline XferPlan xfer_plan(size_t total) {
   return p;
 }
 
+// The pieces of `count` parts of the given bytes, each piece inside one part:
+// their number, and piece i (`at`: the bytes of the pieces before it).  Worked
+// out per piece, not listed: a read through the C interface allocates nothing
+// on the heap but its threads, whose failure it survives.
+struct XferPiece {
+  int part;
+  size_t offset, bytes, at;
+};
+inline size_t xfer_pieces(const size_t* bytes, int count, size_t piece) {
+  size_t n = 0;
+  for (int k = 0; k < count; ++k) n += (bytes[k] + piece - 1) / piece;
+  return n;
+}
+inline XferPiece xfer_piece(const size_t* bytes, int count, size_t piece, size_t i) {
+  size_t at = 0;
+  for (int k = 0; k < count; ++k) {
+    const size_t n = (bytes[k] + piece - 1) / piece;
+    if (i < n) return {k, i * piece, std::min(piece, bytes[k] - i * piece), at + i * piece};
+    i -= n;
+    at += bytes[k];
+  }
+  return {count, 0, 0, at};
+}
+
 }  // namespace mpm

@@ -268,37 +268,37 @@ bool status_failed(const mpm_ctx* ctx) {
 
 // Leaves the stream synchronised.
 int copy_to_host(mpm_ctx* ctx, const XferPart* parts, int count, char* mirror) {
-  struct Piece {
-    char *dst, *via;
-    const char* src;
-    size_t bytes;
-  };
-  std::vector<Piece> pieces;
-  size_t total = 0;
-  for (int k = 0; k < count; ++k) total += parts[k].bytes;
+  constexpr int MOST = 8;
+  if (count > MOST) return MPM_ERR_ARG;
+  size_t bytes[MOST], total = 0;
+  for (int k = 0; k < count; ++k) total += bytes[k] = parts[k].bytes;
   const XferPlan plan = xfer_plan(total);
   const unsigned nt = plan.threads;
-  const size_t piece = plan.piece;
-  size_t at = 0;
-  for (int k = 0; k < count; ++k)
-    for (size_t o = 0; o < parts[k].bytes; o += piece) {
-      const size_t b = std::min(piece, parts[k].bytes - o);
-      pieces.push_back({static_cast<char*>(parts[k].dst) + o, mirror ? mirror + at : nullptr,
-                        static_cast<const char*>(parts[k].src) + o, b});
-      at += b;
-    }
-  if (pieces.empty()) {
+  const size_t pieces = xfer_pieces(bytes, count, plan.piece);
+  if (pieces == 0) {
     IO_HIP(hipStreamSynchronize(ctx->stream));
     return MPM_OK;
   }
   if (int rc = ensure_xfer(ctx, mirror ? 0 : plan.ring)) return rc;
-  if (pieces.size() == 1) {  // nothing to overlap: one wait
-    const Piece& p = pieces[0];
-    char* via = p.via ? p.via : ctx->xfer_host;
-    launch_copy_out(via, p.src, (int64_t)(p.bytes / 4), ctx->stream);
-    IO_HIP(hipGetLastError());
+  // piece i into pinned memory, through ring slot `slot` where there is no
+  // mirror, and from there on
+  auto via = [&](const XferPiece& p, unsigned slot) {
+    return mirror ? mirror + p.at : ctx->xfer_host + slot * plan.piece;
+  };
+  auto put = [&](size_t i, unsigned slot) {
+    const XferPiece p = xfer_piece(bytes, count, plan.piece, i);
+    launch_copy_out(via(p, slot), static_cast<const char*>(parts[p.part].src) + p.offset, (int64_t)(p.bytes / 4),
+                    ctx->stream);
+    return hipGetLastError();
+  };
+  auto take = [&](size_t i, unsigned slot) {
+    const XferPiece p = xfer_piece(bytes, count, plan.piece, i);
+    std::memcpy(static_cast<char*>(parts[p.part].dst) + p.offset, via(p, slot), p.bytes);
+  };
+  if (pieces == 1) {  // nothing to overlap: one wait
+    IO_HIP(put(0, 0));
     IO_HIP(hipStreamSynchronize(ctx->stream));
-    std::memcpy(p.dst, via, p.bytes);
+    take(0, 0);
     return MPM_OK;
   }
   // thread t takes pieces t, t + nt, ... through its two slots
@@ -306,21 +306,13 @@ int copy_to_host(mpm_ctx* ctx, const XferPart* parts, int count, char* mirror) {
   auto work = [&](unsigned t) {
     hipError_t& e = errs[t];
     if (t) e = hipSetDevice(ctx->device);
-    size_t prev = pieces.size();
+    size_t prev = pieces;
     unsigned k = 0;
-    for (size_t i = t; e == hipSuccess && (i < pieces.size() || prev < pieces.size()); i += nt, ++k) {
-      if (i < pieces.size()) {
-        Piece& p = pieces[i];
-        const unsigned slot = 2 * t + (k & 1);
-        if (!p.via) p.via = ctx->xfer_host + slot * piece;
-        launch_copy_out(p.via, p.src, (int64_t)(p.bytes / 4), ctx->stream);
-        if ((e = hipGetLastError()) == hipSuccess) e = hipEventRecord(ctx->xfer_ev[slot], ctx->stream);
-      }
-      if (e == hipSuccess && prev < pieces.size()) {
-        const Piece& p = pieces[prev];
-        e = hipEventSynchronize(ctx->xfer_ev[2 * t + ((k + 1) & 1)]);
-        if (e == hipSuccess) std::memcpy(p.dst, p.via, p.bytes);
-      }
+    for (size_t i = t; e == hipSuccess && (i < pieces || prev < pieces); i += nt, ++k) {
+      const unsigned slot = 2 * t + (k & 1), before = 2 * t + ((k + 1) & 1);
+      if (i < pieces && (e = put(i, slot)) == hipSuccess) e = hipEventRecord(ctx->xfer_ev[slot], ctx->stream);
+      if (e == hipSuccess && prev < pieces && (e = hipEventSynchronize(ctx->xfer_ev[before])) == hipSuccess)
+        take(prev, before);
       prev = i;
     }
   };

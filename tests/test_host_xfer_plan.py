@@ -23,3 +23,26 @@ def test_ring_is_bounded_by_the_copy(total):
     assert 1 <= threads <= 4 and piece % 64 == 0 and 64 <= piece <= 1 << 20
     assert ring >= 2 * threads * piece
     assert ring <= min(8 << 20, max(128, 2 * (total + 64)))
+
+
+@pytest.mark.parametrize("bytes_", [[4], [0, 4, 0], [64, 68, 60], [100, 200, 4], [4 * 2147, 12 * 2147, 36 * 2147, 0, 36 * 2147],
+                                    [12 * 700001, 12 * 700001, 36 * 700001, 36 * 700001, 36 * 700001, 4 * 700001]])
+@pytest.mark.parametrize("piece", [64, 128, 1 << 17, 1 << 20])
+def test_pieces_tile_every_part(bytes_, piece):
+    if sum(bytes_) // piece > 20000:
+        piece = 1 << 20
+    L = C.CDLL(LIB)
+    Z = C.POINTER(C.c_size_t)
+    L.hc_xfer_pieces.argtypes, L.hc_xfer_pieces.restype = [Z, C.c_int, C.c_size_t], C.c_size_t
+    L.hc_xfer_piece.argtypes = [Z, C.c_int, C.c_size_t, C.c_size_t, Z]
+    b = (C.c_size_t * len(bytes_))(*bytes_)
+    part, offset, at = 0, 0, 0
+    for i in range(L.hc_xfer_pieces(b, len(bytes_), piece)):
+        out = (C.c_size_t * 4)()
+        L.hc_xfer_piece(b, len(bytes_), piece, i, out)
+        while offset == bytes_[part]:  # a part's end, or an empty part
+            part, offset = part + 1, 0
+        assert (out[0], out[1], out[3]) == (part, offset, at) and out[1] % 64 == 0
+        assert 0 < out[2] <= piece and offset + out[2] <= bytes_[part]
+        offset, at = offset + out[2], at + out[2]
+    assert at == sum(bytes_)
