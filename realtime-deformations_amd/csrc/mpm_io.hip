@@ -301,11 +301,13 @@ int copy_to_host(mpm_ctx* ctx, const XferPart* parts, int count, char* mirror) {
     take(0, 0);
     return MPM_OK;
   }
-  // thread t takes pieces t, t + nt, ... through its two slots
+  // thread t takes pieces t, t + nt, ... through its two slots; a thread made
+  // here has the context's device to select, the caller's keeps its own
   hipError_t errs[XFER_THREADS] = {};
+  const std::thread::id caller = std::this_thread::get_id();
   auto work = [&](unsigned t) {
     hipError_t& e = errs[t];
-    if (t) e = hipSetDevice(ctx->device);
+    if (std::this_thread::get_id() != caller) e = hipSetDevice(ctx->device);
     size_t prev = pieces;
     unsigned k = 0;
     for (size_t i = t; e == hipSuccess && (i < pieces || prev < pieces); i += nt, ++k) {
