@@ -503,15 +503,15 @@ void launch_adj_p2g(const KArgs& a, const float* St, const float* Gin, float* Go
   // chip stays part empty.  us for a forward and backward of 24 substeps (the
   // first three) and of 40 with checkpoints every 20:
   //                1      2      4
-  //    2,000    2396   2299   2267
-  //    6,000    2582   2492   2456
-  //   20,000    3251   3166   3264
-  //    8,000    4043   3867   3824
-  //   20,011    4497   4326   4488
-  //   32,768    5054   4897   5026
-  //   40,022    5368   5357   5644
-  //   60,033    6298   6243   6732
-  //   98,304    8484   8660   9321
+  //    2,000    2477   2374   2417
+  //    6,000    2745   2640   2598
+  //   20,000    3143   3010   3122
+  //    8,000    4124   3950   3907
+  //   20,011    4428   4259   4427
+  //   32,768    5077   4906   5054
+  //   40,022    5407   5386   5670
+  //   60,033    5863   5943   6338
+  //   98,304    8203   8512   9220
   const int lanes = a.n <= 12000 ? 4 : a.n <= 40000 ? 2 : 1;
   auto k = lanes == 4 ? k_adj_p2g<4> : lanes == 2 ? k_adj_p2g<2> : k_adj_p2g<1>;
   if (a.n) k<<<nblk((int64_t)a.n * lanes), TPB, 0, s>>>(a, St, Gin, Gout, gnode, gE, Sv, SvPrev);

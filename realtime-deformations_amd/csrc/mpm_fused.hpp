@@ -4,12 +4,13 @@
 
 namespace mpm {
 
-// The substep epoch lives on the device, so one captured substep can be
-// replayed as a HIP graph: grid-block lists alternate with the epoch's
-// parity, their counters rotate with it modulo 3.  It takes two words: the
-// block pass reads dstep[0] and copies it to dstep[1]; the grid pass that
-// follows reads dstep[1] and writes dstep[0] = dstep[1] + 1.  No launch
-// writes the word it reads, so neither pass has to find its last workgroup.
+// The substep epoch (BlockArgs.dstep) lives on the device, so one captured
+// substep can be replayed as a HIP graph: grid-block lists alternate with the
+// epoch's parity, their counters rotate with it modulo 3.  It takes two words:
+// the block pass reads dstep[0] and copies it to dstep[1]; the grid pass that
+// follows reads dstep[1] and writes dstep[0] = dstep[1] + 1.  No launch writes
+// the word it reads, so neither pass has to find its last workgroup.
+
 // Reverse-mode record of one substep's grid: the P2G sums of its active
 // grid blocks, 64 nodes each, in the order of list (list[0]: the count,
 // list[1 + s]: the grid block of record slot s).
