@@ -217,25 +217,18 @@ Scene make_scene(const mpm_params& p) {
 // particles at a time, 10 us a round where few are on the chip, and 768
 // workgroups fit it; small contexts have fewer blocks than that, of several
 // rounds each, so their blocks are cut.  A part pays a block's halo (load,
-// clear, flush, this last in FP64) again, so whole blocks are best once they
-// fill the chip: with 8 particles a cell, 500 a block, from 600,000 on, with
-// 15 a cell above 800,000, where the line is.  us for a call, measured on
-// balls and slabs of 8 particles a cell where nothing else is said:
+// clear, flush) again, so whole blocks are best once they fill the chip.
+// us for a call, measured on balls and slabs:
 //                                   whole    256    512    768
-//     8,192 x 20 substeps            1040    523    674    728
-//   131,072 x 32, 15 a cell          3092   2004   2023   2388
-//   200,000 x 20                     1614   1594   1439   1694
-//   262,144 x 32, 15 a cell          3332   2982   2688   2857
-//   400,000 x 20                     2579   2814   2459   2636
-//   500,000 x 20                     2804          2770   2885
-//   524,288 x 48, reverse           22865  23760  21793  21902
-//   600,000 x 20                     3125          3211   3187
-//   600,000 x 32, 15 a cell          4686   5174   4197   4357
-//   800,000 x 20                     3855          3959   3922
-//   800,000 x 32, 15 a cell          5670          5256   5261
-//   1,048,576 x 20                   4538   5410   4665   4724
-//   2,000,000 x 20                   6987   8719   7352   7107
-int work_chunk(int n) { return n <= 160000 ? 256 : n <= 800000 ? 512 : 0; }
+//     8,192 x 20 substeps            1214    537    690
+//   131,072 x 32                     3384   1939   1985
+//   200,000 x 20                     1838   1566   1423
+//   400,000 x 20                     2951   2696   2399
+//   524,288 x 48, 8 a cell, reverse 23298  27728  24296  23050
+//   600,000 x 32, 15 a cell          4804   4739   4132   4235
+//   1,048,576 x 20                   4427   4994   4543   4454
+//   2,000,000 x 20                   6876   8020   7216   7011
+int work_chunk(int n) { return n <= 160000 ? 256 : n <= 450000 ? 512 : n <= 800000 ? 768 : 0; }
 
 int upload_scene_table(mpm_ctx* ctx) {
   MPM_HIP(hipStreamSynchronize(ctx->stream));

@@ -34,7 +34,7 @@ def _same_grids(g, n):
     np.testing.assert_array_equal(b["vel"], a["vel"])
 
 
-# parts of 256 particles, then of 512
+# the three part sizes of 256, 512 and 768
 SIZES = [131072, 262144, 524288]
 
 
