@@ -198,7 +198,11 @@ MPM_HD float rcp_exact(float y) {
   return 1.0f / y;
 #endif
 }
-MPM_HD float div_exact(float a, float b, float r) { return div_rcp(a, b, r); }
+MPM_HD float div_exact(float a, float b, float r) {
+  const float q = a * r;
+  const float e = fmaf(q, b, -a);  // minus div_rcp's residual: for b > 0 a zero a keeps its sign
+  return fmaf(-e, r, q);
+}
 MPM_HD float sqrt_ge1(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const float s = __builtin_amdgcn_sqrtf(x);
@@ -217,8 +221,7 @@ MPM_HD double rcp_unit(double y) { return 1.0 / y; }
 MPM_HD void rcp_pair(float u, float w, float& rw, float& uw) {
   if (fabsf(u) <= 1.15292150e18f) {  // 2^60
     rw = rcp_exact(w);
-    // |u| < 2^-60: w = 1, exact as it is, but for the sign of -0
-    uw = __builtin_copysignf(div_exact(u, w, rw), u);
+    uw = div_exact(u, w, rw);  // |u| < 2^-60: w = 1, exact as it is
   } else {
     rw = 1.0f / w;
     uw = u / w;

@@ -73,5 +73,6 @@ def test_quotients(dev, kind, seed):
     a = np.ldexp(a, ea).astype(np.float32) * rng.choice(np.float32([-1, 1]), a.size)
     b = np.ldexp(b, eb).astype(np.float32) * rng.choice(np.float32([-1, 1]), a.size)
     _same_bits(dev.debug_svd_arith("div", a, b), a / b)
-    zero = np.zeros(4, np.float32)
-    _same_bits(dev.debug_svd_arith("div", zero, np.float32([1, 2, 3, 0.1])), zero)
+    zero = np.float32([0.0, -0.0, 0.0, -0.0])
+    b = np.float32([1, 2, 3, 0.1])  # divisors of a rotation are positive
+    _same_bits(dev.debug_svd_arith("div", zero, b), zero / b)
