@@ -580,22 +580,21 @@ __global__ void __launch_bounds__(TPB, 3) k_block_pass(BlockArgs ba) {
     }
     __syncthreads();
     if (kP2G) {
-      for (int q = t; q < HN * HN * HN; q += TPB) {
-        const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
-        const int l = hx * TX + tile_y(hy) + tile_z(hz);
-        if (EXACT || a.wide) {  // EXACT: exact sums of multiples of the quanta
-          const double m = ah[l], px = ah[TPLANE + l], py = ah[2 * TPLANE + l], pz = ah[3 * TPLANE + l];
-          if (m != 0.0 || px != 0.0 || py != 0.0 || pz != 0.0) {
-            const int gi = o[0] + hx, gj = o[1] + hy, gk = o[2] + hz;
-            if (gi >= 0 && gj >= 0 && gk >= 0 && gi < S.dims[0] && gj < S.dims[1] && gk < S.dims[2]) {
-              double* g = reinterpret_cast<double*>(a.gacc64 + node_index(gi, gj, gk, S));
-              atomicAdd(g + 0, m);
-              atomicAdd(g + 1, px);
-              atomicAdd(g + 2, py);
-              atomicAdd(g + 3, pz);
-            }
-          }
-        } else {
+      if (EXACT || a.wide) {
+        // FP64 (EXACT: exact sums of multiples of the quanta): a lane per node
+        // and component, so that a row of nodes is one run of memory
+        for (int c = t; c < 4 * HN * HN * HN; c += TPB) {
+          const int q = c >> 2, f = c & 3;
+          const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
+          const double u = ah[f * TPLANE + hx * TX + tile_y(hy) + tile_z(hz)];
+          const int gi = o[0] + hx, gj = o[1] + hy, gk = o[2] + hz;
+          if (u != 0.0 && gi >= 0 && gj >= 0 && gk >= 0 && gi < S.dims[0] && gj < S.dims[1] && gk < S.dims[2])
+            atomicAdd(reinterpret_cast<double*>(a.gacc64 + node_index(gi, gj, gk, S)) + f, u);
+        }
+      } else {
+        for (int q = t; q < HN * HN * HN; q += TPB) {
+          const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
+          const int l = hx * TX + tile_y(hy) + tile_z(hz);
           const float m = (float)ah[l], px = (float)ah[TPLANE + l], py = (float)ah[2 * TPLANE + l],
                       pz = (float)ah[3 * TPLANE + l];
           if (m != 0.0f || px != 0.0f || py != 0.0f || pz != 0.0f) {
@@ -801,24 +800,27 @@ __global__ void __launch_bounds__(TPB) k_adj_g2p_block(BlockArgs ba, const float
       for (int k = 0; k < 3; ++k) Gout[(int64_t)(FX + k) * sd + p] = gx[k];
     }
     __syncthreads();
-    for (int q = t; q < HN * HN * HN; q += TPB) {
-      const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
-      const int l = hx * TX + tile_y(hy) + tile_z(hz);
-      const double u0 = gh[l], u1 = gh[TPLANE + l], u2 = gh[2 * TPLANE + l];
-      if (u0 != 0.0 || u1 != 0.0 || u2 != 0.0) {
+    if (gsum) {  // a lane per node and component, as the forward flush
+      for (int c = t; c < 3 * HN * HN * HN; c += TPB) {
+        const int q = c / 3, f = c % 3;
+        const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
+        const double u = gh[f * TPLANE + hx * TX + tile_y(hy) + tile_z(hz)];
         const int gi = o[0] + hx, gj = o[1] + hy, gk = o[2] + hz;
-        if (gi >= 0 && gj >= 0 && gk >= 0 && gi < S.dims[0] && gj < S.dims[1] && gk < S.dims[2]) {
-          const int64_t g = node_index(gi, gj, gk, S);
-          if (gsum) {
-            double* gn = reinterpret_cast<double*>(gsum + g);
+        if (u != 0.0 && gi >= 0 && gj >= 0 && gk >= 0 && gi < S.dims[0] && gj < S.dims[1] && gk < S.dims[2])
+          atomicAdd(reinterpret_cast<double*>(gsum + node_index(gi, gj, gk, S)) + 1 + f, u);
+      }
+    } else {
+      for (int q = t; q < HN * HN * HN; q += TPB) {
+        const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
+        const int l = hx * TX + tile_y(hy) + tile_z(hz);
+        const float u0 = (float)gh[l], u1 = (float)gh[TPLANE + l], u2 = (float)gh[2 * TPLANE + l];
+        if (u0 != 0.0f || u1 != 0.0f || u2 != 0.0f) {
+          const int gi = o[0] + hx, gj = o[1] + hy, gk = o[2] + hz;
+          if (gi >= 0 && gj >= 0 && gk >= 0 && gi < S.dims[0] && gj < S.dims[1] && gk < S.dims[2]) {
+            float* gn = reinterpret_cast<float*>(gnode + node_index(gi, gj, gk, S));
             atomicAdd(gn + 1, u0);
             atomicAdd(gn + 2, u1);
             atomicAdd(gn + 3, u2);
-          } else {
-            float* gn = reinterpret_cast<float*>(gnode + g);
-            atomicAdd(gn + 1, (float)u0);
-            atomicAdd(gn + 2, (float)u1);
-            atomicAdd(gn + 3, (float)u2);
           }
         }
       }
