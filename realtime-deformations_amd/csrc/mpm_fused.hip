@@ -483,6 +483,57 @@ __device__ __forceinline__ void load_halo(float* __restrict__ vh, const float4* 
   }
 }
 
+// FP64 sums of a halo into the grid's: components FIRST to 3 of each node, a
+// plane of the halo each.  A lane per node has its four atomics 32 bytes from
+// the next lane's, so a wave goes over the same lines four times, which binds
+// where many workgroups flush at once; with a lane per node and component a
+// row of nodes is one run of memory, in four times the rounds, which a body on
+// few blocks waits for.  The line lies between bodies of 65 and of 127
+// entries.  us for a call of 20 substeps, a lane per node and per component:
+//   particles (entries)    falling     in a heap
+//     4,000 (34)          484  490     630  648
+//     8,192 (64)          519  492     629  644
+//    16,384 (127)         594  514     664  667
+//    32,768 (236)         678  560     745  708
+//   131,072 (848)        1006  797    1430 1250
+// (100,003 reproducible: 3,020 and 2,560; 3 x 20,011 with gradients: 5,857 and
+// 4,980.)
+constexpr int FLUSH_FEW = 96;
+template <int FIRST>
+__device__ __forceinline__ void flush_sums(const double* __restrict__ h, double4* __restrict__ grid, const Scene& S,
+                                           const int o[3], int nblocks) {
+  constexpr int NODES = HN * HN * HN, N = 4 - FIRST;
+  const int t = threadIdx.x;
+  if (nblocks > FLUSH_FEW) {
+    for (int c = t; c < N * NODES; c += TPB) {
+      const int q = c / N, f = c % N;
+      const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
+      const double u = h[f * TPLANE + hx * TX + tile_y(hy) + tile_z(hz)];
+      const int gi = o[0] + hx, gj = o[1] + hy, gk = o[2] + hz;
+      if (u != 0.0 && gi >= 0 && gj >= 0 && gk >= 0 && gi < S.dims[0] && gj < S.dims[1] && gk < S.dims[2])
+        atomicAdd(reinterpret_cast<double*>(grid + node_index(gi, gj, gk, S)) + FIRST + f, u);
+    }
+    return;
+  }
+  for (int q = t; q < NODES; q += TPB) {
+    const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
+    const int l = hx * TX + tile_y(hy) + tile_z(hz);
+    double u[N];
+    bool any = false;
+#pragma unroll
+    for (int f = 0; f < N; ++f) {
+      u[f] = h[f * TPLANE + l];
+      any = any || u[f] != 0.0;
+    }
+    const int gi = o[0] + hx, gj = o[1] + hy, gk = o[2] + hz;
+    if (any && gi >= 0 && gj >= 0 && gk >= 0 && gi < S.dims[0] && gj < S.dims[1] && gk < S.dims[2]) {
+      double* g = reinterpret_cast<double*>(grid + node_index(gi, gj, gk, S)) + FIRST;
+#pragma unroll
+      for (int f = 0; f < N; ++f) atomicAdd(g + f, u[f]);
+    }
+  }
+}
+
 // BATCHED = 0 (one scene): the scene comes from the kernel arguments,
 // read-only and loop-invariant; BATCHED = 1: each block's scene from the
 // device table, copied once per block into scalar registers.
@@ -580,17 +631,8 @@ __global__ void __launch_bounds__(TPB, 3) k_block_pass(BlockArgs ba) {
     }
     __syncthreads();
     if (kP2G) {
-      if (EXACT || a.wide) {
-        // FP64 (EXACT: exact sums of multiples of the quanta): a lane per node
-        // and component, so that a row of nodes is one run of memory
-        for (int c = t; c < 4 * HN * HN * HN; c += TPB) {
-          const int q = c >> 2, f = c & 3;
-          const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
-          const double u = ah[f * TPLANE + hx * TX + tile_y(hy) + tile_z(hz)];
-          const int gi = o[0] + hx, gj = o[1] + hy, gk = o[2] + hz;
-          if (u != 0.0 && gi >= 0 && gj >= 0 && gk >= 0 && gi < S.dims[0] && gj < S.dims[1] && gk < S.dims[2])
-            atomicAdd(reinterpret_cast<double*>(a.gacc64 + node_index(gi, gj, gk, S)) + f, u);
-        }
+      if (EXACT || a.wide) {  // EXACT: exact sums of multiples of the quanta
+        flush_sums<0>(ah, a.gacc64, S, o, nblocks);
       } else {
         for (int q = t; q < HN * HN * HN; q += TPB) {
           const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
@@ -800,15 +842,8 @@ __global__ void __launch_bounds__(TPB) k_adj_g2p_block(BlockArgs ba, const float
       for (int k = 0; k < 3; ++k) Gout[(int64_t)(FX + k) * sd + p] = gx[k];
     }
     __syncthreads();
-    if (gsum) {  // a lane per node and component, as the forward flush
-      for (int c = t; c < 3 * HN * HN * HN; c += TPB) {
-        const int q = c / 3, f = c % 3;
-        const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
-        const double u = gh[f * TPLANE + hx * TX + tile_y(hy) + tile_z(hz)];
-        const int gi = o[0] + hx, gj = o[1] + hy, gk = o[2] + hz;
-        if (u != 0.0 && gi >= 0 && gj >= 0 && gk >= 0 && gi < S.dims[0] && gj < S.dims[1] && gk < S.dims[2])
-          atomicAdd(reinterpret_cast<double*>(gsum + node_index(gi, gj, gk, S)) + 1 + f, u);
-      }
+    if (gsum) {
+      flush_sums<1>(gh, gsum, S, o, nblocks);
     } else {
       for (int q = t; q < HN * HN * HN; q += TPB) {
         const int hx = q / (HN * HN), hy = (q / HN) % HN, hz = q % HN;
