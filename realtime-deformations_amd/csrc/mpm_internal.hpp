@@ -343,6 +343,9 @@ struct CopyList {
   }
 };
 void launch_copy_list(const CopyList& l, hipStream_t s);
+// the substep epochs from 1 again: block counters (4), epoch words (2) and,
+// since no block is due for zeroing then, BV_STEP
+void launch_reset_epochs(int* gcnt, int* dstep, int* bvars, hipStream_t s);
 void launch_iota(int* p, int n, hipStream_t s);
 void launch_fill_int(int* p, int64_t n, int v, hipStream_t s);
 void launch_grid_to_dense(const KArgs& a, const Scene& S, float* m, float* vel, float* force, uint8_t* active,

@@ -312,6 +312,11 @@ __global__ void __launch_bounds__(256) k_copy_list(CopyList l) {
     }
   }
 }
+__global__ void k_reset_epochs(int* gcnt, int* dstep, int* bvars) {
+  for (int k = 0; k < 4; ++k) gcnt[k] = 0;
+  dstep[0] = dstep[1] = 1;
+  bvars[BV_STEP] = 0;
+}
 __global__ void k_iota(int* p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = i;
@@ -423,6 +428,9 @@ void launch_copy_list(const CopyList& l, hipStream_t s) {
   int64_t most = 0;
   for (int f = 0; f < l.count; ++f) most = std::max(most, l.words[f]);
   if (most > 0) k_copy_list<<<(int)std::min<int64_t>((most / 4 + TPB) / TPB, 4096), TPB, 0, s>>>(l);
+}
+void launch_reset_epochs(int* gcnt, int* dstep, int* bvars, hipStream_t s) {
+  k_reset_epochs<<<1, 1, 0, s>>>(gcnt, dstep, bvars);
 }
 void launch_iota(int* p, int n, hipStream_t s) {
   if (n) k_iota<<<nblk(n), TPB, 0, s>>>(p, n);
