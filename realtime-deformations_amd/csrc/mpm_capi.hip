@@ -217,17 +217,27 @@ Scene make_scene(const mpm_params& p) {
 // particles at a time, 10 us a round where few are on the chip, and 768
 // workgroups fit it; small contexts have fewer blocks than that, of several
 // rounds each, so their blocks are cut.  A part pays a block's halo (load,
-// clear, flush) again, so whole blocks are best once they fill the chip.
-// us for a call, measured on balls and slabs:
-//                                   whole    256    512    768
-//     8,192 x 20 substeps            1214    537    690
-//   131,072 x 32                     3384   1939   1985
-//   200,000 x 20                     1838   1566   1423
-//   400,000 x 20                     2951   2696   2399
-//   524,288 x 48, 8 a cell, reverse 23298  27728  24296  23050
-//   600,000 x 32, 15 a cell          4804   4739   4132   4235
-//   1,048,576 x 20                   4427   4994   4543   4454
-//   2,000,000 x 20                   6876   8020   7216   7011
+// clear, FP64 flush) again, so whole blocks are best once they fill the chip,
+// and beyond 2,048 entries workgroups claim them, an atomic on one address
+// each: the lines lie where bodies of 8 to 10 particles a cell stay below
+// that (the ball of 654,890: its G2P pass takes 27 us with parts of 768, 58
+// with parts of 512).  Between the lines smaller parts gain where cells are
+// fuller.  us for a call, measured on balls and slabs of 8 particles a cell
+// where nothing else is said:
+//                                      whole    256    512    768
+//     8,192 x 20 substeps               1038    496    680    706
+//   131,072 x 32, 15 a cell             3049   1446   1804   2255
+//   200,000 x 20                        1607   1371   1434   1661
+//   262,144 x 32, 15 a cell             3222   2274   2277   2682
+//   400,000 x 20                        2598   2492   2440   2670
+//   500,000 x 20                        2772   2773   2753   2898
+//   524,288 x 48, reverse              22990  21261  20759  21206
+//   600,000 x 32, 15 a cell             4648   4224   3922   4044
+//   654,890 x 2 and a read, 9.7 a cell   535    595    593    529
+//   800,000 x 20                        3782   3917   3922   3944
+//   800,000 x 32, 15 a cell             5649   5128   4909   4893
+//   1,048,576 x 20                      4463   4763   4698   4602
+//   2,000,000 x 20                      6857   7747   7315   7136
 int work_chunk(int n) { return n <= 160000 ? 256 : n <= 450000 ? 512 : n <= 800000 ? 768 : 0; }
 
 int upload_scene_table(mpm_ctx* ctx) {
@@ -749,11 +759,9 @@ void reset_grid(mpm_ctx* ctx) {
   launch_clear(reinterpret_cast<float4*>(ctx->gacc), 2 * ctx->nnodes, s);
   launch_clear(ctx->gvel, ctx->nnodes, s);
   launch_fill_int(ctx->gflag, ctx->nblocks, 0, s);
-  launch_fill_int(ctx->gcnt, 4, 0, s);
-  launch_fill_int(ctx->dstep, 2, 1, s);
   // the epochs start again in a binning made before: BV_STEP is of the old
   // count, and with the velocities cleared no block is due for zeroing
-  launch_fill_int(ctx->bvars + BV_STEP, 1, 0, s);
+  launch_reset_epochs(ctx->gcnt, ctx->dstep, ctx->bvars, s);
   ctx->gacc_clean = true;
 }
 
