@@ -503,15 +503,15 @@ void launch_adj_p2g(const KArgs& a, const float* St, const float* Gin, float* Go
   // chip stays part empty.  us for a forward and backward of 24 substeps (the
   // first three) and of 40 with checkpoints every 20:
   //                1      2      4
-  //    2,000    2477   2374   2417
-  //    6,000    2745   2640   2598
-  //   20,000    3143   3010   3122
-  //    8,000    4124   3950   3907
-  //   20,011    4428   4259   4427
-  //   32,768    5077   4906   5054
-  //   40,022    5407   5386   5670
-  //   60,033    5863   5943   6338
-  //   98,304    8203   8512   9220
+  //    2,000    2562   2470   2414
+  //    6,000    2760   2683   2646
+  //   20,000    3073   2955   3054
+  //    8,000    4086   3930   3889
+  //   20,011    4069   3910   4077
+  //   32,768    4254   4099   4241
+  //   40,022    4440   4450   4724
+  //   60,033    4998   5003   5469
+  //   98,304    6215   6401   7064
   const int lanes = a.n <= 12000 ? 4 : a.n <= 40000 ? 2 : 1;
   auto k = lanes == 4 ? k_adj_p2g<4> : lanes == 2 ? k_adj_p2g<2> : k_adj_p2g<1>;
   if (a.n) k<<<nblk((int64_t)a.n * lanes), TPB, 0, s>>>(a, St, Gin, Gout, gnode, gE, Sv, SvPrev);
