@@ -57,6 +57,24 @@ def test_node_adjoints_are_rounded_once(n):
     g.close()
 
 
+@pytest.mark.parametrize("n", [1, 95 * 256, 95 * 256 + 1])
+def test_both_flushes(n):
+    """At most 96 entries, and one more, where the flush changes its lanes: one
+    rounding of N times the single particle's mass at every node; dL/dv0 within
+    its gather's 64 terms."""
+    g = _pair(n, V)
+    g.init_volumes()
+    g.substeps(1e-4, 1)
+    g.sync()
+    a, b = g.scene_grid(0), g.scene_grid(1)
+    np.testing.assert_array_equal(b["m"], (np.float64(n) * a["m"].astype(np.float64)).astype(np.float32))
+    np.testing.assert_array_equal(b["active"], a["active"])
+    g.adjoint_forward(1e-4, 1, 1)
+    _, gv0, _ = g.adjoint_backward(None, G * np.ones((n + 1, 1), np.float32))
+    assert np.abs(gv0[1:] - gv0[0]).max() <= 64 * 2.0 ** -24 * np.abs(gv0[0]).max()
+    g.close()
+
+
 def test_particles_beyond_their_halo():
     """Six substeps of 0.64 cells without a binning: the last sums come from
     the scatter to global memory.  The reverse sweep's per-lane order of x
